@@ -256,42 +256,78 @@ __global__ __launch_bounds__(64 * W) void rbf_fwd_split_kernel(const Params p) {
   qn2 = c * 0.5f * xhalf_sum(qn2);
   const frag ones = ones_frag<T>();
 
+  constexpr bool STATIC = SOFTMAX && !std::is_same<T, _Float16>::value;
   f32x16_t oacc[ND];
   float x[2];  // sums of the rounded P (normalises O) and of the unrounded P (gives L)
   float m_run;
   auto run = [&](auto safe_tag) {
     constexpr bool SAFE = decltype(safe_tag)::value;
+    // fp16, whose every pass is this one: one offset for the block's waves (bf16
+    // comes here only in the rerun; sharing there too would cost its static pass
+    // 2 %, B1 H16 N1333 D128 28.25 -> 28.93 us, by the compiler's register use)
+    constexpr bool SHARED = SOFTMAX && SAFE && !STATIC;
 #pragma unroll
     for (int d = 0; d < ND; ++d) oacc[d] = zero16();
     x[0] = x[1] = 0.f;
     m_run = !SOFTMAX ? qn2 : (SAFE ? -__builtin_inff() : qn2 - kBoundMargin);
+    float m_all = m_run;  // SHARED: the running maximum over all blocks so far, the same in the block's KSP waves
     split_pipeline(nkt, issue, [&](int kt, int buf) {
       const int k0 = org + 32 * (kt * KSP + ki);
-      if (!wave_on || k0 >= N || !blk_any(q0, k0, causal, npre)) return;
+      const bool on = wave_on && k0 < N && blk_any(q0, k0, causal, npre);
+      if (!SHARED && !on) return;
       const T* kt_ = sT[buf][0] + 32 * ki * DP;
       const T* vt_ = sT[buf][1] + 32 * ki * DP;
-      frag kA[KS];
-#pragma unroll
-      for (int t = 0; t < KS; ++t) kA[t] = ld8<T>(kt_ + L::off(n, 16 * t + 8 * h));
       f32x16_t s = zero16();
-      float kn = 0.f;
-#pragma unroll
-      for (int t = 0; t < KS; ++t) {
-        s = E::mma(kA[t], qf[t], s);
-        kn += sumsq8<T>(kA[t]);
-      }
-      kn = xhalf_sum(kn);
-      s = row_term((k0 + n >= 0 && k0 + n < N) ? -0.5f * kn : -__builtin_inff(), h, s);
       frag vA[ND][2];
+      if (on) {
+        frag kA[KS];
 #pragma unroll
-      for (int d = 0; d < ND; ++d)
+        for (int t = 0; t < KS; ++t) kA[t] = ld8<T>(kt_ + L::off(n, 16 * t + 8 * h));
+        float kn = 0.f;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) vA[d][t] = L::template tr<T>(vt_, 16 * t, 32 * d, lane);
-      if (!blk_nomask(q0, k0, causal, npre)) mask_key_rows(s, k0, h, jmax);
-      if constexpr (SOFTMAX && SAFE) {
+        for (int t = 0; t < KS; ++t) {
+          s = E::mma(kA[t], qf[t], s);
+          kn += sumsq8<T>(kA[t]);
+        }
+        kn = xhalf_sum(kn);
+        s = row_term((k0 + n >= 0 && k0 + n < N) ? -0.5f * kn : -__builtin_inff(), h, s);
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) vA[d][t] = L::template tr<T>(vt_, 16 * t, 32 * d, lane);
+        if (!blk_nomask(q0, k0, causal, npre)) mask_key_rows(s, k0, h, jmax);
+      }
+      if constexpr (SOFTMAX && SAFE && !SHARED) {
         const float mt = xhalf_max(tree_max16(s)) * c;
         if (__any(mt > m_run + kTau)) {
           const float mnew = fmaxf(m_run, mt);
+          const float alpha = (mnew == -__builtin_inff()) ? 1.f : fast_exp2(m_run - mnew);
+#pragma unroll
+          for (int d = 0; d < ND; ++d) oacc[d] *= alpha;
+          x[0] *= alpha;
+          x[1] *= alpha;
+          m_run = mnew;
+        }
+      }
+      if constexpr (SHARED) {
+        // The offset takes the tile's blocks in key order, by the rule and with
+        // the values of the streaming kernel, so that P is rounded to T at the
+        // same scale there and here.  Outputs of the two at B4 H8 N1024 D64:
+        // 2.6e-4 apart (as much as fp16's own error) where a wave went by its own
+        // blocks alone, 0.2e-4 this way; the step's time did not change (65.3 us
+        // before, 60-65 after).
+        const float mt = on ? xhalf_max(tree_max16(s)) * c : -__builtin_inff();
+        if (h == 0) sM[wave][n] = mt;
+        lds_barrier();
+        float mnew = m_run;
+#pragma unroll
+        for (int e = 0; e < KSP; ++e) {
+          const float me = sM[wave - ki + e][n];
+          if (__any(me > m_all + kTau)) m_all = fmaxf(m_all, me);
+          if (e == ki) mnew = m_all;
+        }
+        if (!on) return;
+        if (__any(mnew > m_run)) {
           const float alpha = (mnew == -__builtin_inff()) ? 1.f : fast_exp2(m_run - mnew);
 #pragma unroll
           for (int d = 0; d < ND; ++d) oacc[d] *= alpha;
@@ -318,23 +354,24 @@ __global__ __launch_bounds__(64 * W) void rbf_fwd_split_kernel(const Params p) {
       }
     });
     if constexpr (SOFTMAX && SAFE) {
-      // bring the splits' partials to the block's largest offset
-      if (h == 0) sM[wave][n] = m_run;
-      __syncthreads();
-      float M = m_run;
+      // bring the wave's partials from its last offset to the block's
+      if constexpr (!SHARED) {
+        if (h == 0) sM[wave][n] = m_run;
+        __syncthreads();
+        m_all = m_run;
 #pragma unroll
-      for (int e = 0; e < KSP; ++e) M = fmaxf(M, sM[wave - ki + e][n]);
-      const float w = (m_run == -__builtin_inff()) ? 0.f : fast_exp2(m_run - M);
+        for (int e = 0; e < KSP; ++e) m_all = fmaxf(m_all, sM[wave - ki + e][n]);
+      }
+      const float w = (m_run == -__builtin_inff()) ? 0.f : fast_exp2(m_run - m_all);
 #pragma unroll
       for (int d = 0; d < ND; ++d) oacc[d] *= w;
       x[0] *= w;
       x[1] *= w;
-      m_run = M;
+      m_run = m_all;
     }
     split_sum<W, KSP, ND, 2>(oacc, x, reinterpret_cast<f32x4_t*>(&sT[0][0][0]), sX, wave, lane);
   };
 
-  constexpr bool STATIC = SOFTMAX && !std::is_same<T, _Float16>::value;
   if constexpr (SOFTMAX && !STATIC) run(std::true_type{});
   else run(std::false_type{});
   if constexpr (STATIC) {
