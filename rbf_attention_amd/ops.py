@@ -601,14 +601,22 @@ def rbf_decode(q, k_cache, v_cache, cache_lens=None, *, softmax=True, sm_scale=N
 def _eager_plain(*ts) -> bool:
     """Whether a wrapper call may take the eager path: plain GPU tensors (no
     subclass: fake, functional, distributed ...; no meta or CPU tensors), not
-    under torch.compile / export tracing, no dispatch mode and no functorch
-    transform.  Everything else goes through the registered ops, which those
-    mechanisms know (and which raise for CPU tensors)."""
-    if torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active():
-        return False
-    if _python_dispatch._get_current_dispatch_mode() is not None:
-        return False
-    return all(t is None or (type(t) is torch.Tensor and t.is_cuda) for t in ts)
+    under torch.compile / export tracing or torch.jit.trace, no dispatch mode
+    and no functorch transform.  Everything else goes through the registered
+    ops, which those mechanisms know (and which raise for CPU tensors)."""
+    return _outside_tracing() and all(t is None or (type(t) is torch.Tensor and t.is_cuda) for t in ts)
+
+
+def _outside_tracing() -> bool:
+    """No compiler, tracer, dispatch mode or functorch transform is to see the
+    call.  (torch.jit.trace does not record the native binding's nodes: a trace
+    of them holds only the empty output.)"""
+    return not (
+        torch.compiler.is_compiling()
+        or torch._C._is_tracing()
+        or torch._C._are_functorch_transforms_active()
+        or _python_dispatch._get_current_dispatch_mode() is not None
+    )
 
 
 def run_triton_rbf(q, k, v, is_causal=True, *, sm_scale=None, num_prefix=0, token_major=False, pos=None):

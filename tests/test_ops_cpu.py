@@ -95,3 +95,61 @@ def test_eager_path_predicate():
     # the meta tensors go through the ops' fake implementations
     assert ra.run_triton_rbf(m, m, m).shape == m.shape
     assert ra.run_triton_non_softmax_rbf(m, m, m, sm_scale=0.1, num_prefix=2).shape == m.shape
+
+
+def _stand_in(softmax):
+    """Plain torch forward and backward with the ops' implementations' signatures."""
+
+    def scores(q, k, causal, g, npre):
+        s = 2 * g * (q @ k.transpose(-1, -2)) - g * (k * k).sum(-1).unsqueeze(-2)
+        if not softmax:
+            s = s - g * (q * q).sum(-1, keepdim=True)
+        n = q.shape[2]
+        i = torch.arange(n)
+        return s.masked_fill(~((i <= i[:, None]) | (i < npre) | (not causal)), float("-inf"))
+
+    def fwd(q, k, v, causal, g, npre, token_major=False, pos=None):
+        q, k = (q, k) if pos is None else (q + pos, k + pos)
+        s = scores(q, k, causal, g, npre)
+        return (s.softmax(-1) @ v, s.logsumexp(-1)) if softmax else s.exp() @ v
+
+    def bwd(q, k, v, *rest):
+        do, causal, g, npre = rest[2:6] if softmax else rest[:4]
+        s = scores(q, k, causal, g, npre)
+        p = s.softmax(-1) if softmax else s.exp()
+        ds = p * (do @ v.transpose(-1, -2))
+        if softmax:
+            ds = ds - p * ds.sum(-1, keepdim=True)
+        dq = 2 * g * (ds @ k - (0 if softmax else ds.sum(-1, keepdim=True) * q))
+        return dq, 2 * g * (ds.transpose(-1, -2) @ q - ds.sum(-2).unsqueeze(-1) * k), p.transpose(-1, -2) @ do
+
+    return fwd, bwd
+
+
+@pytest.mark.parametrize("softmax", [True, False])
+@pytest.mark.parametrize("kw", [{}, {"sm_scale": 0.3, "num_prefix": 2}])
+def test_jit_trace(monkeypatch, softmax, kw):
+    """Under torch.jit.trace no call takes the eager path, and the ops are
+    recorded: a traced call's values and gradients are the eager ones."""
+    from rbf_attention_amd import ops
+
+    fwd, bwd = _stand_in(softmax)
+    monkeypatch.setattr(ops, "_softmax_fwd" if softmax else "_non_softmax_fwd", fwd)
+    monkeypatch.setattr(ops, "_softmax_bwd" if softmax else "_non_softmax_bwd", bwd)
+    fn = ra.run_triton_rbf if softmax else ra.run_triton_non_softmax_rbf
+    seen = []
+
+    def call(q, k, v):
+        seen.append(ops._outside_tracing())
+        return fn(q, k, v, True, **kw)
+
+    gen = torch.Generator().manual_seed(1)
+    new = lambda: [torch.randn(1, 2, 9, 8, generator=gen).requires_grad_() for _ in range(3)]  # noqa: E731
+    traced = torch.jit.trace(call, new())
+    assert not seen[0] and ops._outside_tracing()  # later calls: the tracer checks its trace against the function
+    x = new()
+    want, got = call(*x), traced(*x)
+    torch.testing.assert_close(got, want)
+    do = torch.randn(want.shape, generator=gen)
+    for a, b in zip(torch.autograd.grad(got, x, do), torch.autograd.grad(want, x, do)):
+        torch.testing.assert_close(a, b)
