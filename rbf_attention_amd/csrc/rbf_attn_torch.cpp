@@ -25,6 +25,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -187,10 +188,13 @@ std::tuple<Tensor, Tensor, Tensor> backward(Tensor q, Tensor k, const Tensor& v,
 }
 
 // The packed (B, N, 3, H, D) tensor of which q, k and v, in this order, are the
-// (B, H, N, D) views; undefined if they are not.
+// (B, H, N, D) views; undefined if they are not, or if anything else refers to
+// their memory (a gradient that a hook kept, that autograd.grad returns, or a
+// view of one): a gradient is never shared with another.
 Tensor packed_of(const Tensor& q, const Tensor& k, const Tensor& v) {
   if (!q.defined() || !k.defined() || !v.defined() || q.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes() ||
-      !q.is_alias_of(k) || !q.is_alias_of(v) || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type())
+      !q.is_alias_of(k) || !q.is_alias_of(v) || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() ||
+      q.use_count() != 1 || k.use_count() != 1 || v.use_count() != 1 || q.storage().use_count() != 3)
     return Tensor();
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3);
   const int64_t strides[4] = {N * 3 * H * D, D, 3 * H * D, 1};
@@ -204,8 +208,8 @@ Tensor packed_of(const Tensor& q, const Tensor& k, const Tensor& v) {
 // Autograd of select or unbind stacks the three gradients and then copies the
 // stack to this layout for the projection's backward (38 + 37 us of a 670 us
 // module step at B32 N516 H8 D64); this node's backward returns the packed
-// tensor itself when the attention's backward wrote the three into one (below),
-// and else copies each into its place.
+// tensor itself when the attention's backward wrote the three into one (below)
+// and they are referred to nowhere else, and else copies each into its place.
 struct UnpackFunction : torch::autograd::Function<UnpackFunction> {
   static variable_list forward(AutogradContext* ctx, const Variable& qkv) {
     ctx->saved_data["sizes"] = qkv.sizes().vec();
@@ -233,18 +237,27 @@ struct UnpackFunction : torch::autograd::Function<UnpackFunction> {
   }
 };
 
-// Whether q, k and v are the three outputs of one UnpackFunction.
-bool unpacked_together(const Tensor& q, const Tensor& k, const Tensor& v) {
+// Whether the gradients of q, k and v go to one UnpackFunction that will use them
+// up, so that a packed tensor of the three pays: q, k and v are its outputs, this
+// backward pass runs it, and no hook and no autograd.grad asks for them there (a
+// dq that is kept would keep the memory of all three).
+bool pack_gradients(const Tensor& q, const Tensor& k, const Tensor& v) {
   if (!q.requires_grad() || !k.requires_grad() || !v.requires_grad()) return false;
   const auto& f = q.grad_fn();
-  return f && f == k.grad_fn() && f == v.grad_fn() && q.output_nr() == 0 && k.output_nr() == 1 && v.output_nr() == 2 &&
-         dynamic_cast<torch::autograd::CppNode<UnpackFunction>*>(f.get()) != nullptr;
+  if (!f || f != k.grad_fn() || f != v.grad_fn() || q.output_nr() != 0 || k.output_nr() != 1 || v.output_nr() != 2 ||
+      dynamic_cast<torch::autograd::CppNode<UnpackFunction>*>(f.get()) == nullptr)
+    return false;
+  if (!f->pre_hooks().empty() || !f->tensor_pre_hooks().empty() || !f->retains_grad_hooks().empty()) return false;
+  const auto* info = torch::autograd::get_current_graph_task_exec_info();
+  if (info == nullptr || info->empty()) return true;  // a pass that runs every node
+  const auto it = info->find(f.get());
+  return it != info->end() && it->second.needed_ && !it->second.captures_;
 }
 
 struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
   static Variable forward(AutogradContext* ctx, const Variable& q, const Variable& k, const Variable& v,
                           const std::optional<Variable>& pos, bool softmax, bool causal, double scale, int64_t num_prefix,
-                          bool token_major, bool packed) {
+                          bool token_major) {
     const Call c = {softmax, causal, token_major, scale, num_prefix};
     const Tensor p = pos.has_value() ? *pos : Tensor();
     auto [out, L] = ::forward(q, k, v, p, c);
@@ -254,7 +267,6 @@ struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["num_prefix"] = num_prefix;
-    ctx->saved_data["packed"] = packed;
     return out;
   }
 
@@ -262,11 +274,13 @@ struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
     const Call c = {ctx->saved_data["softmax"].toBool(), ctx->saved_data["causal"].toBool(), false,
                     ctx->saved_data["scale"].toDouble(), ctx->saved_data["num_prefix"].toInt()};
     const variable_list s = ctx->get_saved_variables();
-    // As the registered backward ops: the result carries no graph of its own.
-    const at::NoGradGuard no_grad;
     const Tensor& q = s[0];
+    const bool pack = q.size(3) % 8 == 0 && pack_gradients(q, s[1], s[2]);
+    // As the registered backward ops: the result carries no graph of its own, and
+    // the views of a packed tensor no record of their base.
+    const at::AutoDispatchBelowADInplaceOrView below_autograd;
     Tensor packed;
-    if (ctx->saved_data["packed"].toBool() && q.size(3) % 8 == 0)
+    if (pack)
       packed = at::empty({q.size(0), q.size(2), 3, q.size(1), q.size(3)}, q.options());
     auto [dq, dk, dv] =
         ::backward(q, s[1], s[2], c.softmax ? s[4] : Tensor(), c.softmax ? s[5] : Tensor(), grads[0], s[3], c, packed);
@@ -276,7 +290,7 @@ struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
       at::add_out(dpos, dq, dk);
       if (s[3].size(0) == 1 && dpos.size(0) != 1) dpos = dpos.sum(0, /*keepdim=*/true);
     }
-    return {dq, dk, dv, dpos, Variable(), Variable(), Variable(), Variable(), Variable(), Variable()};
+    return {dq, dk, dv, dpos, Variable(), Variable(), Variable(), Variable(), Variable()};
   }
 };
 
@@ -324,8 +338,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Tensor out;
   {
     const pybind11::gil_scoped_release no_gil;
-    out = RbfAttentionFunction::apply(q, k, v, pos, softmax, causal, scale, (int64_t)num_prefix, token_major,
-                                      unpacked_together(q, k, v));
+    out = RbfAttentionFunction::apply(q, k, v, pos, softmax, causal, scale, (int64_t)num_prefix, token_major);
   }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS

@@ -1,7 +1,8 @@
 """The packed gradient of q, k and v (ops.unpack_qkv) against plain views of the
 same projection output, bit for bit: the attention's own gradients, with one of
 the three used elsewhere too (its gradient is then a sum), with one unused, and
-with gradients asked for at the views."""
+with gradients asked for at the views.  A gradient that a program gets hold of
+shares its memory with no other."""
 import pytest
 import torch
 
@@ -51,3 +52,93 @@ def test_packed_gradient_with_a_graph(cuda_device):
         (h,) = torch.autograd.grad((g * g).sum(), x)
         got.append((g.detach(), h))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def inputs(dev, B=2, N=40, H=2, D=64):
+    g = torch.Generator().manual_seed(5)
+    qkv = torch.randn(B, N, 3, H, D, generator=g).to(dev, torch.bfloat16)
+    return qkv, torch.randn(B, H, N, D, generator=g).to(dev, torch.bfloat16)
+
+
+def shares(a, b):
+    return a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr()
+
+
+def test_gradient_kept_by_a_hook(cuda_device):
+    """A leaf's gradient is added to in place by the next backward pass; what a
+    hook kept of the first pass stays what it was."""
+    qkv, do = inputs(cuda_device)
+    x = qkv.clone().requires_grad_(True)
+    for keep in (lambda g: g, lambda g: g[0], lambda g: g.detach()):
+        kept = []
+        x.grad = None
+        for _ in range(2):
+            q, k, v = ops.unpack_qkv(x)
+            if not kept:
+                q.register_hook(lambda g: kept.append((keep(g), g.clone())))
+            ra.run_triton_rbf(q, k, v).backward(do)
+        view, copy = kept[0]
+        assert torch.equal(view, copy if view.dim() == 4 else copy[0])
+        assert not shares(view, x.grad)
+
+
+@pytest.mark.parametrize("at", ["tensor", "node", "attention_node"])
+def test_gradient_kept_by_node_hooks(cuda_device, at):
+    qkv, do = inputs(cuda_device)
+    x = qkv.clone().requires_grad_(True)
+    q, k, v = ops.unpack_qkv(x)
+    out = ra.run_triton_rbf(q, k, v)
+    kept = []
+    if at == "tensor":
+        q.retain_grad()
+        v.register_hook(kept.append)
+    elif at == "node":
+        q.grad_fn.register_prehook(lambda grads: kept.extend(grads))
+    else:
+        out.grad_fn.register_hook(lambda grad_inputs, _: kept.extend(grad_inputs[:3]))
+    out.backward(do)
+    assert kept and not any(shares(g, x.grad) for g in kept)
+    if at == "tensor":
+        assert not shares(q.grad, x.grad)
+        # and a kept dv holds its own memory only
+        assert kept[0].untyped_storage().nbytes() == kept[0].numel() * kept[0].element_size()
+
+
+@pytest.mark.parametrize("ask", ["q", "q_x", "x_q_k_v"])
+def test_gradients_asked_for_together(cuda_device, ask):
+    """autograd.grad at the views and at the packed tensor: writing to one result
+    leaves the others alone, each holds its own memory, and the values are those
+    of plain views."""
+    qkv, do = inputs(cuda_device)
+    results = []
+    for split in (ops.unpack_qkv, lambda t: t.permute(2, 0, 3, 1, 4).unbind(0)):
+        x = qkv.clone().requires_grad_(True)
+        q, k, v = split(x)
+        wrt = {"q": (q,), "q_x": (q, x), "x_q_k_v": (x, q, k, v)}[ask]
+        results.append(torch.autograd.grad(ra.run_triton_rbf(q, k, v), wrt, do))
+    ours, plain = results
+    assert all(torch.equal(a, b) for a, b in zip(ours, plain))
+    for i, g in enumerate(ours):
+        assert g.untyped_storage().nbytes() == g.numel() * g.element_size()
+        others = [o.clone() for j, o in enumerate(ours) if j != i]
+        g.zero_()
+        assert all(torch.equal(o, c) for o, c in zip((o for j, o in enumerate(ours) if j != i), others))
+
+
+def test_packed_gradient_is_not_copied(cuda_device):
+    """Nothing else asks for dq, dk and dv: one buffer is written, no other of its
+    size is allocated."""
+    qkv, do = inputs(cuda_device, 8, 256, 8, 64)
+    x = qkv.clone().requires_grad_(True)
+    peaks = []
+    for split in (ops.unpack_qkv, lambda t: t.permute(2, 0, 3, 1, 4).unbind(0)):
+        for _ in range(2):  # the first pass loads kernels
+            x.grad = None
+            out = ra.run_triton_rbf(*split(x))
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            base = torch.cuda.memory_allocated()
+            out.backward(do)
+            peak = torch.cuda.max_memory_allocated() - base
+        peaks.append(peak / x.nbytes)
+    assert peaks[0] < 1.2 and peaks[1] > 1.9, peaks
