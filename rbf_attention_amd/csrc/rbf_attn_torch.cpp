@@ -21,6 +21,7 @@
 #include <vector>
 
 #include <ATen/ATen.h>
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
@@ -220,7 +221,11 @@ struct UnpackFunction : torch::autograd::Function<UnpackFunction> {
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const auto first = std::find_if(grads.begin(), grads.end(), [](const Tensor& g) { return g.defined(); });
     if (first == grads.end()) return {Variable()};
-    if (at::GradMode::is_enabled()) {  // create_graph: a gradient that has a graph of its own
+    // create_graph (a gradient that has a graph of its own), or gradients of
+    // another kind than the attention's (batched by vmap, subclasses)
+    if (at::GradMode::is_enabled() || std::any_of(grads.begin(), grads.end(), [](const Tensor& g) {
+          return g.defined() && at::isTensorSubclassLike(g);
+        })) {
       std::vector<Tensor> parts;
       for (const Tensor& g : grads) parts.push_back((g.defined() ? g : at::zeros_like(*first)).transpose(1, 2));
       return {at::stack(parts, 2)};
@@ -350,6 +355,7 @@ PyObject* unpack_qkv(PyObject*, PyObject* o) {
   if (!THPVariable_Check(o)) Py_RETURN_NONE;
   const Tensor& qkv = unpack(o);
   if (qkv.dim() != 5 || qkv.size(2) != 3 || !qkv.is_contiguous()) Py_RETURN_NONE;
+  if (qkv._fw_grad(/*level=*/0).defined()) Py_RETURN_NONE;  // forward mode: plain views have it
   const variable_list v = UnpackFunction::apply(qkv);
   PyObject* r = PyTuple_New(3);
   if (r == nullptr) return nullptr;

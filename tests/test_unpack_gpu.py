@@ -142,3 +142,22 @@ def test_packed_gradient_is_not_copied(cuda_device):
             peak = torch.cuda.max_memory_allocated() - base
         peaks.append(peak / x.nbytes)
     assert peaks[0] < 1.2 and peaks[1] > 1.9, peaks
+
+
+def test_forward_mode_and_batched_gradients(cuda_device):
+    """As plain views: tangents of a dual tensor, and a batch of gradients."""
+    import torch.autograd.forward_ad as fwad
+
+    g = torch.Generator().manual_seed(3)
+    x, t = (torch.randn(2, 5, 3, 2, 8, generator=g).to(cuda_device) for _ in range(2))
+    cot = torch.randn(4, 2, 2, 5, 8, generator=g).to(cuda_device)
+    results = []
+    for split in (ops.unpack_qkv, lambda t: t.permute(2, 0, 3, 1, 4).unbind(0)):
+        with fwad.dual_level():
+            q, k, v = split(fwad.make_dual(x, t))
+            tangent = fwad.unpack_dual(q * k + v).tangent
+        leaf = x.clone().requires_grad_(True)
+        q, k, v = split(leaf)
+        (batch,) = torch.autograd.grad(q * k + v, leaf, cot, is_grads_batched=True)
+        results.append((tangent, batch))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
