@@ -259,6 +259,30 @@ bool pack_gradients(const Tensor& q, const Tensor& k, const Tensor& v) {
   return it != info->end() && it->second.needed_ && !it->second.captures_;
 }
 
+bool like(const Tensor& t, const Tensor& q) {
+  return t.scalar_type() == q.scalar_type() && t.device() == q.device();
+}
+
+// What the backward pass reads, as the registered backward ops check it: the
+// saved tensors may have gone through a program's saved-tensor hooks, which can
+// bring them back in another shape, type or place.
+void check_saved(const Tensor& q, const variable_list& others, const Tensor& pos, const Tensor& L) {
+  TORCH_CHECK_VALUE(q.dim() == 4 && q.size(3) <= 256, "scaled_bwd: expected (B, H, N, D) tensors, got q of shape ", q.sizes());
+  TORCH_CHECK_TYPE(dtype_code(q.scalar_type()) >= 0, "scaled_bwd: unsupported dtype ", q.scalar_type());
+  TORCH_CHECK(q.is_cuda(), "scaled_bwd: the RBF attention kernels run only on a ROCm GPU, tensors are on ", q.device());
+  const auto check = [&](const Tensor& t, at::IntArrayRef sizes, at::ScalarType type) {
+    TORCH_CHECK_VALUE(t.sizes() == sizes, "scaled_bwd: shape mismatch ", t.sizes(), " vs ", sizes);
+    TORCH_CHECK_TYPE(t.scalar_type() == type, "scaled_bwd: dtype mismatch ", t.scalar_type(), " vs ", type);
+    TORCH_CHECK_VALUE(t.device() == q.device(), "scaled_bwd: device mismatch ", t.device(), " vs ", q.device());
+  };
+  for (const Tensor& t : others) check(t, q.sizes(), q.scalar_type());
+  if (L.defined()) check(L, q.sizes().slice(0, 3), at::kFloat);
+  if (pos.defined()) {
+    const int64_t sizes[4] = {pos.dim() == 4 && pos.size(0) == 1 ? 1 : q.size(0), q.size(1), q.size(2), q.size(3)};
+    check(pos, sizes, q.scalar_type());
+  }
+}
+
 struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
   static Variable forward(AutogradContext* ctx, const Variable& q, const Variable& k, const Variable& v,
                           const std::optional<Variable>& pos, bool softmax, bool causal, double scale, int64_t num_prefix,
@@ -280,6 +304,9 @@ struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
                     ctx->saved_data["scale"].toDouble(), ctx->saved_data["num_prefix"].toInt()};
     const variable_list s = ctx->get_saved_variables();
     const Tensor& q = s[0];
+    variable_list others = {s[1], s[2], grads[0]};
+    if (c.softmax) others.push_back(s[4]);
+    check_saved(q, others, s[3], c.softmax ? s[5] : Tensor());
     const bool pack = q.size(3) % 8 == 0 && pack_gradients(q, s[1], s[2]);
     // As the registered backward ops: the result carries no graph of its own, and
     // the views of a packed tensor no record of their base.
@@ -288,7 +315,7 @@ struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
     if (pack)
       packed = at::empty({q.size(0), q.size(2), 3, q.size(1), q.size(3)}, q.options());
     auto [dq, dk, dv] =
-        ::backward(q, s[1], s[2], c.softmax ? s[4] : Tensor(), c.softmax ? s[5] : Tensor(), grads[0], s[3], c, packed);
+        ::backward(q, s[1], s[2], c.softmax ? s[4] : Tensor(), c.softmax ? s[5].contiguous() : Tensor(), grads[0], s[3], c, packed);
     Tensor dpos;
     if (s[3].defined()) {
       dpos = at::empty(dq.sizes(), dq.options());
@@ -301,9 +328,6 @@ struct RbfAttentionFunction : torch::autograd::Function<RbfAttentionFunction> {
 
 bool takes_dims(const Tensor& q) {
   return q.dim() == 4 && q.is_cuda() && dtype_code(q.scalar_type()) >= 0 && q.size(3) >= 1 && q.size(3) <= 256;
-}
-bool like(const Tensor& t, const Tensor& q) {
-  return t.scalar_type() == q.scalar_type() && t.device() == q.device();
 }
 // a position term (1 or B, H, N, D) of q's type and device
 bool takes_pos(const Tensor& p, const Tensor& q) {
