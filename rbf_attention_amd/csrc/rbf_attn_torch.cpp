@@ -51,10 +51,12 @@ int dtype_code(at::ScalarType t) {
 int64_t padded_dim(int64_t d) { return d <= 8 ? 8 : (d + 7) / 8 * 8; }
 
 // The C ABI's layout contract: unit last stride, 16-byte aligned base and
-// strides, head dim a multiple of 8.  Copies only when needed.
+// strides, head dim a multiple of 8, the values in memory (no negative bit, no
+// tensor of implied zeros).  Copies only when needed.
 Tensor prep(const Tensor& t, int64_t dp) {
   const int64_t d = t.size(3);
   if (dp != d) return at::constant_pad_nd(t, {0, dp - d});
+  if (t.is_neg() || t._is_zerotensor()) return t.clone(at::MemoryFormat::Contiguous);
   const bool base = reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   if (base && t.is_contiguous()) return t;
   const int64_t es = t.element_size();

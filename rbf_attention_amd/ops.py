@@ -70,10 +70,13 @@ def _padded_dim(d: int) -> int:
 
 def _prep(t: torch.Tensor, dpad: int) -> torch.Tensor:
     """Meet the C-ABI layout contract: unit last stride, 16-byte aligned base
-    and strides, head dim a multiple of 8.  Copies only when needed."""
+    and strides, head dim a multiple of 8, the values in memory (no negative
+    bit).  Copies only when needed."""
     d = t.shape[-1]
     if dpad != d:
         return torch.nn.functional.pad(t, (0, dpad - d))
+    if t.is_neg():
+        return t.clone(memory_format=torch.contiguous_format)
     if t.is_contiguous() and t.data_ptr() % 16 == 0:
         return t  # strides are multiples of d, a multiple of 8 elements
     esz = t.element_size()

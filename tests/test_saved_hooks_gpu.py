@@ -1,5 +1,6 @@
 """Saved-tensor hooks around the wrappers: the backward pass checks what the hooks
-bring back before a kernel reads it, and takes any layout."""
+bring back before a kernel reads it, and takes any layout.  And views whose
+memory holds the negated values."""
 import pytest
 import torch
 
@@ -67,3 +68,20 @@ def test_other_layouts(cuda_device, softmax, pos):
         results.append([t.grad for t in x] + ([p.grad] if pos else []))
     for r in results[1:]:
         assert all(torch.equal(a, b) for a, b in zip(r, results[0]))
+
+
+def test_negative_views(cuda_device):
+    """As inputs and as the output's gradient, through the wrapper, the op and the
+    autograd.Function alias."""
+    x, _, do, _ = make(cuda_device, True, False)
+    neg = lambda t: torch._neg_view(-t.detach())  # noqa: E731
+    for fn in (ra.run_triton_rbf, lambda *a: torch.ops.rbf_attn_v5.scaled_fwd(*a, True)[0], ra.TritonRBFAttention.apply):
+        results = []
+        for view in (lambda t: t.detach(), neg):
+            leaves = [view(t).requires_grad_() for t in x]
+            out = fn(*leaves)
+            results.append([out.detach(), *torch.autograd.grad(out, leaves, view(do))])
+        assert all(torch.equal(a, b) for a, b in zip(*results))
+    q, k, v = (t.detach() for t in x)
+    for a, b in zip(ra.rbf_decode(q[:, :, :2], k, v), ra.rbf_decode(neg(q[:, :, :2]), neg(k), neg(v))):
+        assert torch.equal(a, b)
