@@ -192,7 +192,7 @@ def load(path: str | None = None):
 def torch_binding(pos_launcher):
     """The native eager path (_rbf_attn_torch, csrc/rbf_attn_torch.cpp), loaded
     once, after the library that it calls; pos_launcher launches its calls with
-    a fused position term."""
+    a fused position term.  Failed library calls raise RbfAttnError there too."""
     global _torch_binding
     if _torch_binding is None:
         load()
@@ -204,7 +204,7 @@ def torch_binding(pos_launcher):
                 spec = importlib.util.spec_from_file_location("_rbf_attn_torch", path)
                 module = importlib.util.module_from_spec(spec)
                 spec.loader.exec_module(module)
-                module.set_pos_launcher(pos_launcher)
+                module.configure(RbfAttnError, pos_launcher)
                 _torch_binding = module
     return _torch_binding
 

@@ -76,7 +76,32 @@ void* current_stream(const at::Device& dev) {
   return static_cast<void*>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream());
 }
 
-void check_rc(int rc) { TORCH_CHECK(rc == 0, "librbfattn: ", rc, ": ", rbf_attn_last_error()); }
+// Python objects of the ops layer, set once, at load (configure): the error class
+// of failed library calls, and the launcher of calls with a fused position term
+// (ops._launch_pos_bytes: entry point's name, args as bytes, term), the one place
+// where such calls can be observed from Python.
+PyObject* error_class = nullptr;
+PyObject* pos_launcher = nullptr;
+
+// Throws the pending Python error, kept in the exception (it may be caught on
+// another thread, or after the GIL was released).  With the GIL held.
+[[noreturn]] void throw_python_error() {
+  python_error e;
+  e.persist();
+  throw e;
+}
+
+// A failed library call raises _lib.RbfAttnError(code, message).
+void check_rc(int rc) {
+  if (rc == 0) return;
+  const pybind11::gil_scoped_acquire gil;
+  TORCH_CHECK(error_class != nullptr, "librbfattn: ", rc, ": ", rbf_attn_last_error());
+  if (PyObject* e = PyObject_CallFunction(error_class, "is", rc, rbf_attn_last_error())) {
+    PyErr_SetObject(error_class, e);
+    Py_DECREF(e);
+  }
+  throw_python_error();
+}
 
 struct Call {
   bool softmax, causal, token_major;
@@ -112,17 +137,12 @@ void place_pos(const rbf_attn_args& a, Tensor& q, Tensor& k, Tensor& pos, int64_
   }
 }
 
-// The ops layer's launcher of calls with a fused position term
-// (ops._launch_pos_bytes: entry point's name, args as bytes, term), the one
-// place where such calls can be observed from Python.  Set once, at load.
-PyObject* pos_launcher = nullptr;
-
 void launch_pos(const char* name, const rbf_attn_args& a, const Tensor& pos) {
   const pybind11::gil_scoped_acquire gil;
   TORCH_CHECK(pos_launcher != nullptr, "rbf_attn: the position term's launcher is not set");
   PyObject* t = THPVariable_Wrap(pos);
   PyObject* r = PyObject_CallFunction(pos_launcher, "sy#N", name, reinterpret_cast<const char*>(&a), (Py_ssize_t)sizeof(a), t);
-  if (r == nullptr) throw python_error();
+  if (r == nullptr) throw_python_error();
   Py_DECREF(r);
 }
 
@@ -454,14 +474,35 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-PyObject* set_pos_launcher(PyObject*, PyObject* fn) {
-  Py_INCREF(fn);
-  Py_XSETREF(pos_launcher, fn);
+// configure(error class, position term's launcher)
+PyObject* configure(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 2) {
+    PyErr_SetString(PyExc_TypeError, "configure: 2 arguments");
+    return nullptr;
+  }
+  Py_INCREF(args[0]);
+  Py_XSETREF(error_class, args[0]);
+  Py_INCREF(args[1]);
+  Py_XSETREF(pos_launcher, args[1]);
   Py_RETURN_NONE;
 }
 
+// check(code): what a library call that returns this code does
+PyObject* check(PyObject*, PyObject* code) {
+  HANDLE_TH_ERRORS
+  const long rc = PyLong_AsLong(code);
+  if (PyErr_Occurred()) return nullptr;
+  {
+    const pybind11::gil_scoped_release no_gil;
+    check_rc((int)rc);
+  }
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
-    {"set_pos_launcher", set_pos_launcher, METH_O, nullptr},
+    {"configure", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(configure)), METH_FASTCALL, nullptr},
+    {"check", check, METH_O, nullptr},
     {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(attention)), METH_FASTCALL, nullptr},
     {"unpack_qkv", unpack_qkv, METH_O, nullptr},
     {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(decode)), METH_FASTCALL, nullptr},

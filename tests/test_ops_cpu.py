@@ -153,3 +153,15 @@ def test_jit_trace(monkeypatch, softmax, kw):
     do = torch.randn(want.shape, generator=gen)
     for a, b in zip(torch.autograd.grad(got, x, do), torch.autograd.grad(want, x, do)):
         torch.testing.assert_close(a, b)
+
+
+def test_binding_raises_the_library_error():
+    """A library call that fails on the eager path raises RbfAttnError with its
+    code, as the ops do."""
+    from rbf_attention_amd import _lib, ops
+
+    binding = _lib.torch_binding(ops._launch_pos_bytes)
+    assert binding.check(0) is None
+    with pytest.raises(_lib.RbfAttnError) as e:
+        binding.check(-2)
+    assert e.value.code == -2
