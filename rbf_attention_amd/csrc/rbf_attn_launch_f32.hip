@@ -26,6 +26,10 @@ int64_t blocks(const Params& p) { return (int64_t)p.B * p.H * p.nblk; }
 //   the same, all visible    112 / 50 / 77          138 / 68 / 102        160 / 120 / 104 / 136
 //   B8 H8 N1024 (2048)       143 / 60 / 77          178 / 79 / 101        209 / 143 / 122 / 131
 //   B8 H16 N2000 (8064)      943 / 402 / 362        1128 / 549 / 501      1426 / 1022 / 845 / 685
+// Up to 32 features the same limits hold (us fwd / dQ / dK/dV, against the fp32-MFMA
+// kernels, which they stay well below on both sides of each): B1 H8 N300 23 / 28 / 33
+// -> 11 / 13 / 13, B4 H8 N1000 62 / 77 / 96 -> 32 / 38 / 43, B8 H16 N1500 206 / 288 /
+// 360 -> 149 / 184 / 253, B16 H16 N1000 all visible 341 / 480 / 620 -> 244 / 304 / 434.
 // With 128 features a wave's fragments and accumulators leave one wave per
 // SIMD: four-wave work-groups, two waves per block up to 640 blocks (B2 H8 N700
 // 83 -> 55, 98 -> 65, 124 -> 86; at B4 H8 N1500 171 -> 197, 200 -> 230, 256 ->

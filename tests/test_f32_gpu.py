@@ -2,11 +2,15 @@
 float64 oracle, at the edges of their tiles, head-dim widths and of the block
 counts at which the launchers change the split.
 
-Bound beside the max-abs <= 1e-4 of tests/test_parity_gpu.py: relative 2-norm
-<= 2e-5.  An exponential's argument is an fp32 sum of terms up to ~2^6 in base 2
-here, so it carries up to ~2^-18 = 4e-6 of rounding, which is the relative
-error of P; dS adds the rounding of dP - Delta, whose terms cancel by a few
-times, and the products' own sums add 2^-24 per term.
+Bounds beside the max-abs <= 1e-4 of tests/test_parity_gpu.py, on the relative
+2-norm (REL).  An exponential's argument is an fp32 sum of terms up to ~2^6 in base
+2 here, so it carries up to ~2^-18 = 4e-6 of rounding (typically a quarter of it),
+which is the relative error of P; dS adds the rounding of dP - Delta, whose terms
+cancel by a few times, and the products' own sums add 2^-24 per term.  Measured on
+these cases: O up to 0.81e-6, dQ 1.92e-6, dK 2.0e-6, dV 1.85e-6, as with plain fp32
+matrix instructions.  The bounds lie just above, below what the loss of any one
+of the kernels' six part products gives (tests/test_f32_parts_cpu.py: from 1.9e-6,
+2.6e-6, 3.0e-6 and 2.2e-6 on, each beside the rounding above).
 """
 import math
 
@@ -16,6 +20,8 @@ import torch
 from test_parity_gpu import compare_case, np64, oracle_all, rand_inputs
 
 pytestmark = pytest.mark.gpu
+
+REL = {"O": 1.5e-6, "dQ": 2.5e-6, "dK": 2.5e-6, "dV": 2.25e-6}
 
 # (B, H, N, D, softmax, causal, num_prefix)
 CASES = [
@@ -55,7 +61,7 @@ def test_fp32(cuda_device, case):
             for name, got, ref in zip(("O", "dQ", "dK", "dV"), outs, refs):
                 d = np64(got[sl]) - ref
                 rel = float((d ** 2).sum() ** 0.5 / max((ref ** 2).sum() ** 0.5, 1e-30))
-                assert rel <= 2e-5, (name, rel)
+                assert rel <= REL[name], (name, rel)
 
 
 @pytest.mark.parametrize("shift", [3.9, 6.0])
