@@ -78,7 +78,7 @@ struct SLayout {
 // costs one add per instruction.  Tokens outside [0, N) and features >= D read
 // zeros: lanes of such features start at offset 2^31, past every buffer range
 // and, with a tile's row offset added, below 2^32 (the host keeps
-// (N + ROWS) * stride * sizeof(T) within 2^31, dma_split_ok).
+// (N + ROWS) * stride * sizeof(T) within 2^31, split_rows_ok).
 template <typename T, int ROWS, int DP, int W>
 struct DmaRows {
   static_assert(sizeof(T) == 2 && ROWS % 16 == 0, "DMA tiles: 16-bit, whole swizzle periods");
@@ -116,10 +116,10 @@ struct DmaRows {
 
 // s + x[row] for every element of the 32x32 accumulator s, where lane (n, h)
 // gives the x of row n: x = x0 + x1 + x2 with bf16 x0, x1, x2 (24 significant
-// bits cut into three of 8, each exact; -inf stays -inf), multiplied by ones
-// as three contraction indices of one MFMA.
+// bits cut into three of 8, each exact; infinities and NaN stay what they are),
+// multiplied by ones as three contraction indices of one MFMA.
 __device__ __forceinline__ f32x16_t row_term(float x, int h, f32x16_t s) {
-  const bool fin = x > -__builtin_inff();
+  const bool fin = (__float_as_uint(x) & 0x7fffffffu) < 0x7f800000u;
   const uint32_t b0 = __float_as_uint(x) & 0xffff0000u;
   const float r0 = fin ? x - __uint_as_float(b0) : 0.f;
   const uint32_t b1 = __float_as_uint(r0) & 0xffff0000u;
