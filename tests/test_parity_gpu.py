@@ -303,10 +303,10 @@ def test_masks(cuda_device, causal, num_prefix, softmax):
      (64, 4300, torch.bfloat16, False, True, 300), (64, 4300, torch.float16, True, True, 4)],
 )
 def test_masks_long(cuda_device, D, N, dtype, softmax, causal, num_prefix):
-    """Non-causal and register-token masks on the long-sequence streaming
-    kernels with LDS-DMA tiles (D = 128: paired dK/dV kernel; D = 64: DMA
-    dK/dV from N = 4096), whose query-tile ranges start at the first tile when
-    keys are visible to every query."""
+    """Non-causal and register-token masks on one long head (few enough
+    32-token blocks for the split kernels; many heads: test_streaming_gpu),
+    whose query-tile ranges start at the first tile when keys are visible to
+    every query."""
     q, k, v, do = rand_inputs(1, 1, N, D, dtype, cuda_device, std=1.0 if softmax else 0.5, seed=N + D + num_prefix)
     compare_case(q, k, v, do, softmax=softmax, causal=causal, num_prefix=num_prefix, gamma=1.0 / (2 * math.sqrt(D)),
                  tag=f"mask long D{D} N{N} {dtype} sm{softmax} c{causal} p{num_prefix}")
@@ -326,7 +326,8 @@ def test_queries_far_from_every_key(cuda_device, dtype, shift):
     (shift 6) powers of two below the forward's static logit bound
     c*0.5*||q||^2.  The first case stays on the static offset with row sums
     near 2^-40; the second drops below 2^-60 and makes those work-groups
-    recompute with an online max."""
+    recompute with an online max.  (The split kernels' and, in fp32, the fp32
+    kernels'; the streaming kernels' rerun is in test_streaming_gpu.)"""
     q, k, v, do = rand_inputs(2, 4, 200, 64, dtype, cuda_device, seed=17)
     q = q.clone()
     q[:, ::2, :90] += shift
@@ -435,15 +436,12 @@ def test_strided_views_like_the_model(cuda_device):
      (64, 700, torch.bfloat16, True), (64, 4200, torch.bfloat16, True), (64, 4200, torch.float16, False)],
 )
 def test_strided_views_dma_tiles(cuda_device, D, N, dtype, softmax):
-    """q/k/v as views of one packed projection and a permuted dout, for the
-    streaming kernels whose tiles are staged by LDS-DMA (16-bit, D = 64 or
-    128) through buffer resources whose row pitch is the view's token stride
-    (3 H D, or H D for dout); rows past N (N not a multiple of the 64-row
-    tile) read zeros.  D = 128: N = 300 takes the binned short-sequence
-    kernels, N = 2113 the long-sequence ones (paired dK/dV kernel); D = 64
-    (B * H below the CU count, so no head-resident kernels): N = 700 DMA
-    forward and dQ, N = 4200 also the DMA dK/dV.  Checked on the first and
-    the last (b, h) slice."""
+    """q/k/v as views of one packed projection and a permuted dout, for kernels
+    whose tiles are staged by LDS-DMA (16-bit) through buffer resources whose
+    row pitch is the view's token stride (3 H D, or H D for dout); rows past N
+    (N not a multiple of the tile's rows) read zeros.  These six heads take the
+    split kernels at every length here; the streaming kernels' views are in
+    test_streaming_gpu.  Checked on the first and the last (b, h) slice."""
     B, H = 2, 3
     g = torch.Generator().manual_seed(N)
     qkv = (torch.randn(B, N, 3 * H * D, generator=g) * (1.0 if softmax else 0.5)).to(dtype).to(cuda_device)

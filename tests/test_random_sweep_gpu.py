@@ -8,7 +8,9 @@ dimension at once from one fixed generator, so that combinations the fixed
 tests leave out (a padded head dim with a long prefix, fp16 with a
 non-causal mask at a ragged length, strided inputs with D = 24, ...) run
 through whichever kernels the launchers pick for them.  Sizes stay where the
-oracle finishes in about a second (N <= 2000, B * H <= 9).  A second draw
+oracle finishes in about a second (N <= 2000, B * H <= 9), where the 16-bit
+cases take the split kernels (test_streaming_gpu runs the same shapes as one head
+of many, through the streaming kernels).  A second draw
 takes the head-resident kernels (B * H >= 256 heads of N <= 576 tokens,
 32 < D <= 64), compared on sampled (b, h) slices.
 

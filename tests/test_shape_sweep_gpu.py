@@ -1,11 +1,10 @@
 """Parity against the float64 oracle on shapes that straddle the launchers'
 dispatch boundaries, each checked to the bounds of test_parity_gpu:
 
-  * head-resident kernels up to N = 576 at 32 < D <= 64, streaming above;
-  * paired dK/dV kernel at D = 128, with LDS-DMA tile staging from
-    N = 2048 and register staging below (D = 128 exactly; padded head dims
-    such as 96 or 120 always stage through registers);
-  * D = 64 forward and dQ with LDS-DMA at every length, dK/dV from N = 4096;
+  * head-resident kernels up to N = 576 at 32 < D <= 64 where there is a head
+    for every CU, else split kernels for few 32-token blocks (all but one of
+    the 16-bit cases here), streaming above (test_streaming_gpu);
+  * lengths at and around the streaming kernels' own limits;
   * head dims padded to 32 / 64 / 128 (24, 40, 96, 120);
   * B*H not a multiple of 8 (no per-XCD head chunks), B*H = 1;
   * num_prefix register tokens, non-causal masks, fp16 and fp32.
@@ -27,17 +26,17 @@ BF, FP, F32 = torch.bfloat16, torch.float16, torch.float32
 CASES = [
     (1, 3, 577, 64, BF, True, True, 0, "bench"),  # one block past the head-resident limit
     (2, 8, 576, 64, BF, True, True, 4, "ref"),  # at the limit, fewer heads than CUs
-    (1, 2, 2047, 128, BF, True, True, 0, "bench"),  # paired dK/dV, register staging
-    (1, 2, 2048, 128, BF, False, True, 0, "bench"),  # paired dK/dV, LDS-DMA from here on
-    (3, 3, 4095, 64, FP, True, False, 0, "ref"),  # D = 64 forward with DMA, dK/dV without
-    (1, 3, 4096, 64, BF, False, True, 40, "bench"),  # D = 64 dK/dV with DMA, long prefix
-    (5, 3, 1000, 96, BF, True, True, 0, "ref"),  # D = 96 padded to 128
+    (1, 2, 2047, 128, BF, True, True, 0, "bench"),  # D = 128, an odd length
+    (1, 2, 2048, 128, BF, False, True, 0, "bench"),  # D = 128, whole blocks
+    (3, 3, 4095, 64, FP, True, False, 0, "ref"),  # D = 64, one token short of whole blocks
+    (1, 3, 4096, 64, BF, False, True, 40, "bench"),  # D = 64, long prefix
+    (5, 3, 1000, 96, BF, True, True, 0, "ref"),  # D = 96
     (2, 5, 2500, 120, FP, True, True, 0, "bench"),  # D = 120 padded to 128, long
     (1, 1, 3000, 40, BF, False, False, 0, "bench"),  # D = 40 padded to 64, one head
     (4, 4, 300, 24, BF, True, True, 7, "ref"),  # D = 24 padded to 32
     (1, 2, 1500, 128, F32, True, True, 0, "ref"),  # fp32, D = 128
-    (9, 1, 2100, 128, BF, True, True, 0, "bench"),  # B*H = 9, D = 128 DMA
-    (16, 1, 700, 64, BF, True, True, 0, "bench"),  # 16 heads, streaming D = 64
+    (9, 1, 2100, 128, BF, True, True, 0, "bench"),  # B*H = 9, D = 128
+    (16, 1, 700, 64, BF, True, True, 0, "bench"),  # 16 heads, D = 64
     (1, 2, 6000, 64, BF, False, True, 0, "bench"),  # long non-softmax, every DMA path
 ]
 
