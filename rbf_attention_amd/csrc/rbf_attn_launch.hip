@@ -225,9 +225,9 @@ int split_ways(const Params& p, bool dkdv, int64_t stride_a, int64_t stride_b) {
 #endif
 
 // LDS-DMA tile staging (16-bit: the streaming kernels' tiles go from global
-// memory straight into LDS, two or three buffers), when the rows of both operands a kernel stages are ones
-// dma_rows_ok admits (rbf_attn_staging.h); otherwise the kernel is the
-// register-staged one.  Each kernel checks only what it stages: the forward
+// memory straight into LDS, two or three buffers), when the rows of both
+// operands a kernel stages are ones dma_rows_ok admits (rbf_attn_staging.h);
+// otherwise the kernel is the register-staged one.  Each kernel checks only what it stages: the forward
 // and dQ kernels stage K and V (and read Q and dO directly), the dK/dV kernels
 // Q and dO (and read K and V directly); a forward's dO descriptor is unset.
 // RBF_ATTN_DMA=0 keeps the register-staged kernels for every shape.
@@ -322,11 +322,13 @@ hipError_t fwd_default(const Params& p, hipStream_t st) {
     // 367, bf16 345 / 328 / 337.
     if (use_dma_kv(p, DP))
       return p.N >= 1500 ? fwd_cfg<DP, SM, 8, 64, false, 3>(p, st) : fwd_cfg<DP, SM, 4, 64, false, 2>(p, st);
-    // Register staging (D <= 32, or strides past the DMA range): one
-    // group per work-group, 4 waves over 64-key tiles up to N = 8192.
-    // Measured against the binned forms at D = 48 (bf16 softmax fwd, us): B63
-    // H8 N1028 149 -> 117, B20 H8 N700 26.9 -> 23.5, B16 H8 N2052 111 -> 103;
-    // at B4 H8 N8196 the binned 8-wave form stays ahead (360 against 366).
+    // Rows that the LDS-DMA does not take (dma_rows_ok: overlapping, repeated, or
+    // 2^31 bytes of them), through registers: one group per work-group, 4 waves
+    // over 64-key tiles up to N = 8192.  Measured against the binned forms on the
+    // D = 48 rows that came this way before padded head dims took the DMA (bf16
+    // softmax fwd, us): B63 H8 N1028 149 -> 117, B20 H8 N700 26.9 -> 23.5, B16 H8
+    // N2052 111 -> 103; at B4 H8 N8196 the binned 8-wave form stays ahead (360
+    // against 366).
     if (p.N >= 4 * kLongSeq) return bins_fit(p) ? fwd_cfg<DP, SM, 8, 128, true>(p, st) : fwd_cfg<DP, SM, 8, 128>(p, st);
     return fwd_cfg<DP, SM, 4, 64>(p, st);
   } else {
@@ -378,8 +380,8 @@ hipError_t dq_default(const Params& p, hipStream_t st) {
     // -> 168, B16 H8 N1028 45.0 -> 43.2, B20 H8 N700 33.5 -> 31.4, B16 H8
     // N2052 140 -> 126, B15 H8 N4100 491 -> 419, B4 H8 N8196 450 -> 414.
     if (use_dma_kv(p, DP)) return dq_cfg<DP, SM, 4, 1, 64, true, false, 3>(p, st);
-    // register staging: one group per work-group (D = 48: 1.0-4.7 % faster
-    // than binned at N = 700-8196)
+    // rows that the LDS-DMA does not take: one group per work-group (the D = 48
+    // rows that came this way: 1.0-4.7 % faster than binned at N = 700-8196)
     return dq_cfg<DP, SM, 4, 1, 128>(p, st);
   }
   else {
@@ -396,6 +398,8 @@ hipError_t dq_default(const Params& p, hipStream_t st) {
       return p.causal && bins_fit(p) ? dq_cfg<DP, SM, 8, 1, 64, true, true, 3>(p, st)
                                      : dq_cfg<DP, SM, 8, 1, 64, true, false, 3>(p, st);
     }
+    // Rows that the LDS-DMA does not take, through registers (short heads, before
+    // these had a DMA form of their own: B63 H16 N516 302 -> 258 against 8 waves).
     if (p.N < 1200) return dq_cfg<DP, SM, 4, 1, 32, false>(p, st);
     return bins_fit(p) ? dq_cfg<DP, SM, 8, 1, 32, true, true>(p, st) : dq_cfg<DP, SM, 8, 1, 32>(p, st);
   }
@@ -424,17 +428,18 @@ hipError_t dkdv_default(const Params& p, hipStream_t st) {
     // 32 x 256 accumulator
     return dkdv_pair_cfg<DP, SM, 2, 64>(p, st);
   } else if constexpr (DP <= 64) {
-    // LDS-DMA from N = 4096 on: at N = 512-2048 the D = 64 dK/dV measured as
-    // fast or slower with it (C4 188 -> 191 us), at N = 8192 faster (605 -> 589).
-    // With it, one group per work-group (as the forward and dQ): 0.7-3.4 %
-    // faster than the binned form at B15 H8 N4100, B4 H8 N8196, B2 H8 N16388.
-    // From N = 1400 four waves over 64-query tiles of two buffers: 172 -> 164 us
-    // (B16 H8 N2052 non-softmax), 176 -> 169 (softmax), against register-staged
-    // 128-query tiles; 63 -> 64.5 at B16 H8 N1028.
+    // LDS-DMA from N = 1400 on, one group per work-group (as the forward and dQ:
+    // 0.7-3.4 % faster than the binned form at B15 H8 N4100, B4 H8 N8196, B2 H8
+    // N16388).  Below N = 4096 four waves over 64-query tiles of two buffers, 172
+    // -> 164 us (B16 H8 N2052 non-softmax), 176 -> 169 (softmax) against
+    // register-staged 128-query tiles, 63 -> 64.5 at B16 H8 N1028; above, eight
+    // waves over 128-query tiles of three (605 -> 589 at N = 8192 against register
+    // staging, where B16 H8 N2052 takes 188 -> 191).
     if (p.N >= 1400 && use_dma_qdo(p, DP))
       return p.N >= 2 * kLongSeq ? dkdv_cfg<DP, SM, 8, 1, 128, true, false, false, false, 3>(p, st)
                                  : dkdv_cfg<DP, SM, 4, 1, 64, true, false, false, false, 2>(p, st);
-    // Register staging: one group per work-group, 4 waves below N = 4096 and 8
+    // Register staging (shorter heads, and rows that the LDS-DMA does not take): one
+    // group per work-group, 4 waves below N = 4096 and 8
     // above.  Against the binned forms at D = 48 (bf16 softmax dK/dV, us): B63
     // H8 N1028 208 -> 200, B20 H8 N700 38.1 -> 35.9, B16 H8 N2052 169 -> 160,
     // B4 H8 N8196 536 -> 528.
@@ -442,7 +447,7 @@ hipError_t dkdv_default(const Params& p, hipStream_t st) {
     return dkdv_cfg<DP, SM, 4, 1, 128, false>(p, st);
   } else {
     // Four key blocks per work-group, one group each (no bin loop), at every
-    // length; LDS-DMA from N = 1024.  Measured against the binned two-block
+    // length; LDS-DMA up to 96 features, and from N = 1024 above.  Measured against the binned two-block
     // form (bf16 softmax dK/dV): B32 H8 N516 156 -> 114 us, B63 H16 N516 657
     // -> 470, B31 H16 N1028 891 -> 562 (DMA; 585 without), B4 H16 N1500 193
     // -> 114; at B2 H8 N300 18.5 against 18.8.
@@ -620,8 +625,9 @@ hipError_t dkdv_256(const Params& p, bool sm, hipStream_t st) {
 #endif
 
 // Head dim D (a multiple of 8 in [8, 256]) runs on the kernel for the next
-// padded width DP in {32, 64, 128, 256}; features D..DP-1 are zero-filled (as
-// the reference pads to BLOCK_DMODEL = next_pow2(D), rbf_attention.py:661).
+// padded width DP in {32, 64, 128, 256}, of which the streaming kernels of the 128
+// class have a form of 96 features for D <= 96; features D..DP-1 are zero-filled
+// (as the reference pads to BLOCK_DMODEL = next_pow2(D), rbf_attention.py:661).
 // Only the softmax bf16 path with D in (32, 128] carries tuning candidates.
 #define RBF_DISPATCH(DEF, ANY, W256)                                                \
   do {                                                                              \
