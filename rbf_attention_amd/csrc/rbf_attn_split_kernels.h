@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64 * W) void rbf_fwd_split_kernel(const Params p) {
   typedef SLayout<DP> L;
   constexpr int KS = DP / 16, ND = DP / 32, GB = W / KSP, ROWS = 32 * KSP;
   __shared__ __attribute__((aligned(1024))) T sT[2][2][ROWS * DP];
-  __shared__ float sM[W][32];
+  __shared__ float sM[2][W][32];  // the waves' row maxima of a tile, by the tile's parity
   __shared__ float sX[W / 2][2][64];
   static_assert(W / 2 * ND * 4096 <= (int)sizeof(sT), "the partials fit the tiles");
 
@@ -270,33 +270,46 @@ __global__ __launch_bounds__(64 * W) void rbf_fwd_split_kernel(const Params p) {
     for (int d = 0; d < ND; ++d) oacc[d] = zero16();
     x[0] = x[1] = 0.f;
     m_run = !SOFTMAX ? qn2 : (SAFE ? -__builtin_inff() : qn2 - kBoundMargin);
-    float m_all = m_run;  // SHARED: the running maximum over all blocks so far, the same in the block's KSP waves
+    // SHARED: the offset after all blocks so far, the same in the block's KSP waves.
+    // take() moves it over the first `upto` blocks of a tile, in key order and by the
+    // streaming kernel's rule, by the maxima that the waves left in sM (a second time
+    // over the same blocks changes nothing).
+    float m_all = m_run;
+    auto maxima = [&](int par, float (&me)[KSP]) {
+#pragma unroll
+      for (int e = 0; e < KSP; ++e) me[e] = sM[par][wave - ki + e][n];
+    };
+    auto take = [&](const float (&me)[KSP], int upto) {
+#pragma unroll
+      for (int e = 0; e < KSP; ++e)
+        if (e < upto && __any(me[e] > m_all + kTau)) m_all = fmaxf(m_all, me[e]);
+    };
     split_pipeline(nkt, issue, [&](int kt, int buf) {
       const int k0 = org + 32 * (kt * KSP + ki);
       const bool on = wave_on && k0 < N && blk_any(q0, k0, causal, npre);
+      float me[KSP];
+      if constexpr (SHARED) maxima((kt - 1) & 1, me);
       if (!SHARED && !on) return;
       const T* kt_ = sT[buf][0] + 32 * ki * DP;
       const T* vt_ = sT[buf][1] + 32 * ki * DP;
+      frag kA[KS];
+#pragma unroll
+      for (int t = 0; t < KS; ++t) kA[t] = ld8<T>(kt_ + L::off(n, 16 * t + 8 * h));
       f32x16_t s = zero16();
-      frag vA[ND][2];
-      if (on) {
-        frag kA[KS];
+      float kn = 0.f;
 #pragma unroll
-        for (int t = 0; t < KS; ++t) kA[t] = ld8<T>(kt_ + L::off(n, 16 * t + 8 * h));
-        float kn = 0.f;
-#pragma unroll
-        for (int t = 0; t < KS; ++t) {
-          s = E::mma(kA[t], qf[t], s);
-          kn += sumsq8<T>(kA[t]);
-        }
-        kn = xhalf_sum(kn);
-        s = row_term((k0 + n >= 0 && k0 + n < N) ? -0.5f * kn : -__builtin_inff(), h, s);
-#pragma unroll
-        for (int d = 0; d < ND; ++d)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) vA[d][t] = L::template tr<T>(vt_, 16 * t, 32 * d, lane);
-        if (!blk_nomask(q0, k0, causal, npre)) mask_key_rows(s, k0, h, jmax);
+      for (int t = 0; t < KS; ++t) {
+        s = E::mma(kA[t], qf[t], s);
+        kn += sumsq8<T>(kA[t]);
       }
+      kn = xhalf_sum(kn);
+      s = row_term((k0 + n >= 0 && k0 + n < N) ? -0.5f * kn : -__builtin_inff(), h, s);
+      frag vA[ND][2];
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) vA[d][t] = L::template tr<T>(vt_, 16 * t, 32 * d, lane);
+      if (!blk_nomask(q0, k0, causal, npre)) mask_key_rows(s, k0, h, jmax);
       if constexpr (SOFTMAX && SAFE && !SHARED) {
         const float mt = xhalf_max(tree_max16(s)) * c;
         if (__any(mt > m_run + kTau)) {
@@ -310,24 +323,36 @@ __global__ __launch_bounds__(64 * W) void rbf_fwd_split_kernel(const Params p) {
         }
       }
       if constexpr (SHARED) {
-        // The offset takes the tile's blocks in key order, by the rule and with
-        // the values of the streaming kernel, so that P is rounded to T at the
-        // same scale there and here.  Outputs of the two at B4 H8 N1024 D64:
-        // 2.6e-4 apart (as much as fp16's own error) where a wave went by its own
-        // blocks alone, 0.2e-4 this way; the step's time did not change (65.3 us
-        // before, 60-65 after).
+        // So that P is rounded to T at the same scale as in the streaming kernel, its
+        // offset is that kernel's: of all blocks up to this one.  In the first tile,
+        // where they all raise it, the waves wait for one another's maxima; later an
+        // earlier block of the same tile that raises it (by more than kTau) is
+        // seen one tile late.  Outputs of the two kernels at B4 H8 N1024 D64: 2.6e-4
+        // apart (as much as fp16's own error) where a wave went by its own blocks
+        // alone, 0.2e-4 this way.  Times (us; own blocks alone / this / a barrier in
+        // every tile / the streaming kernel): B4 H8 N1024 D64 17.8 / 19.5 / 19.5 / 22.3,
+        // B1 H4 N8000 D64 98 / 107 / 113 / 140, B1 H4 N4000 D128 56 / 60 / 64 / 125.
         const float mt = on ? xhalf_max(tree_max16(s)) * c : -__builtin_inff();
-        if (h == 0) sM[wave][n] = mt;
-        lds_barrier();
+        if (h == 0) sM[kt & 1][wave][n] = mt;
         float mnew = m_run;
+        bool moved = true;
+        if (kt == 0) {
+          lds_barrier();
+          maxima(0, me);
+          take(me, ki + 1);
+          mnew = m_all;
+        } else {
+          float most = mt;
 #pragma unroll
-        for (int e = 0; e < KSP; ++e) {
-          const float me = sM[wave - ki + e][n];
-          if (__any(me > m_all + kTau)) m_all = fmaxf(m_all, me);
-          if (e == ki) mnew = m_all;
+          for (int e = 0; e < KSP; ++e) most = fmaxf(most, me[e]);
+          moved = __any(most > m_all + kTau);
+          if (moved) {
+            take(me, KSP);
+            mnew = __any(mt > m_all + kTau) ? fmaxf(m_all, mt) : m_all;
+          }
         }
         if (!on) return;
-        if (__any(mnew > m_run)) {
+        if (moved) {
           const float alpha = (mnew == -__builtin_inff()) ? 1.f : fast_exp2(m_run - mnew);
 #pragma unroll
           for (int d = 0; d < ND; ++d) oacc[d] *= alpha;
@@ -355,12 +380,17 @@ __global__ __launch_bounds__(64 * W) void rbf_fwd_split_kernel(const Params p) {
     });
     if constexpr (SOFTMAX && SAFE) {
       // bring the wave's partials from its last offset to the block's
-      if constexpr (!SHARED) {
-        if (h == 0) sM[wave][n] = m_run;
+      if constexpr (SHARED) {
+        lds_barrier();
+        float me[KSP];
+        maxima((nkt - 1) & 1, me);
+        take(me, KSP);
+      } else {
+        if (h == 0) sM[0][wave][n] = m_run;
         __syncthreads();
         m_all = m_run;
 #pragma unroll
-        for (int e = 0; e < KSP; ++e) m_all = fmaxf(m_all, sM[wave - ki + e][n]);
+        for (int e = 0; e < KSP; ++e) m_all = fmaxf(m_all, sM[0][wave - ki + e][n]);
       }
       const float w = (m_run == -__builtin_inff()) ? 0.f : fast_exp2(m_run - m_all);
 #pragma unroll
