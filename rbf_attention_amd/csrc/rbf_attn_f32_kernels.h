@@ -211,8 +211,10 @@ __device__ __forceinline__ Frag3 tr3(const __bf16* t, int tbase, int fbase, int 
 // after another, in fp32 on the VALU: scores in LDS, operands read from global
 // memory as they are used, and the output rows themselves as accumulators (element
 // e of a block always by the same thread).  Written for few registers (it is part of
-// kernels whose loops need them), not for speed.  A masked pair is left out, so that
-// an infinity reaches only what it is visible to.
+// kernels whose loops need them), not for speed: a step with an infinite key value in
+// every head takes 13 ms instead of 0.22 at B4 H8 N1001 D64 (accumulators in registers
+// and scores formed once: 8 ms, but the loops' dK/dV 2-7 % slower).  A masked pair is
+// left out, so that an infinity reaches only what it is visible to.
 // ---------------------------------------------------------------------------
 constexpr int kExactRow = 33;  // floats per row of 32 scores in LDS
 
