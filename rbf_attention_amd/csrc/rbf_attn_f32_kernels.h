@@ -41,8 +41,10 @@
 //   B8 H16 N1500 D32   206 / 288 / 360 -> 149 / 184 / 253  0.75 1.68 1.92 1.95 -> 0.75 1.64 1.83 1.81
 // The B8 H16 N2000 D64 forward issues 393 GFLOP of bf16 MFMA in 374 us, 1.05
 // PFLOP/s: bound by the matrix units (a large bf16 matrix product runs at 1.18
-// on the same kind of card).  The lifts and the finite check cost 1-4 % of these
-// times (D = 32 dK/dV 9 %: 233 -> 253).
+// on the same kind of card).  Rounding the high part, the lifts and the finite
+// check cost, over 14 shapes of 16 to 128 features, 2.2 / 3.3 / 6.5 % at the median
+// (fwd / dQ / dK/dV) and 9 / 8 / 14 % at most: B4 H8 N1000 D32 29.3 -> 32.0 and 37.9
+// -> 43.0 (fwd, dK/dV), B1 H8 N300 D32 11.8 -> 12.7 (dQ).
 #pragma once
 
 #include "rbf_attn_kernels.h"
@@ -212,8 +214,9 @@ __device__ __forceinline__ Frag3 tr3(const __bf16* t, int tbase, int fbase, int 
 // memory as they are used, and the output rows themselves as accumulators (element
 // e of a block always by the same thread).  Written for few registers (it is part of
 // kernels whose loops need them), not for speed: a step with an infinite key value in
-// every head takes 13 ms instead of 0.22 at B4 H8 N1001 D64 (accumulators in registers
-// and scores formed once: 8 ms, but the loops' dK/dV 2-7 % slower).  A masked pair is
+// every head takes 13 ms instead of 0.22 at B4 H8 N1001 D64 and 67 instead of 0.72 at
+// B4 H8 N1500 D128 (accumulators in registers and scores formed once: 8 and 30 ms, but
+// the loops' dK/dV 2-7 % slower).  A masked pair is
 // left out, so that an infinity reaches only what it is visible to.
 // ---------------------------------------------------------------------------
 constexpr int kExactRow = 33;  // floats per row of 32 scores in LDS
